@@ -1,0 +1,57 @@
+"""Training backward on inputs whose rows or channels are many powers of two apart,
+row by row against autograd through the float64 recurrence."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+import oracle
+from gdt2_tilelang_amd import chunk_gdn2_bwd
+
+pytestmark = pytest.mark.gpu
+
+NAMES = ("dq", "dk", "dv", "dg", "db", "dw", "dS0")
+
+
+def _inputs(S, H, DK, DV, decay, seed):
+    q, k, v, g, b, w = oracle.make_inputs(1, S, H, DK, DV, decay_scale=decay, seed=seed)
+    gen = torch.Generator().manual_seed(seed + 1)
+    s0, dh = (0.3 * torch.randn(1, H, DK, DV, generator=gen) for _ in range(2))
+    return [q, k, v, g, b, w], s0, torch.randn(1, S, H, DV, generator=gen), dh
+
+
+def _grads64(ins, s0, do, dh):
+    ts = [t.double().requires_grad_(True) for t in (*ins, s0)]
+    o, sf = oracle.recurrent_gdn2(*ts[:6], None, ts[6], True, dtype=torch.float64)
+    return torch.autograd.grad((o, sf), ts, (do.double(), dh.double()))
+
+
+def _grads(ins, s0, do, dh):
+    got = chunk_gdn2_bwd(*(t.cuda() for t in ins), None, *(t.cuda() for t in (s0, do, dh)))
+    torch.cuda.synchronize()
+    return [t.double().cpu() for t in got]
+
+
+def _row_errors(a, r, floor):
+    """Error of each row relative to the row itself, rows below ``floor`` left out."""
+    n = r.norm(dim=-1)
+    return ((a - r).norm(dim=-1) / n)[n > floor]
+
+
+@pytest.mark.parametrize("DK,DV", [(32, 32), (64, 48), (128, 64)])
+@pytest.mark.parametrize("S,decay", [(5, 4.0), (64, 8.0), (130, 8.0), (64, 30.0)])
+def test_state_gradient_by_channel(S, decay, DK, DV):
+    """A channel's row of dS_0 is as small as the decay of its first tokens, down to
+    2^-80 here, and as exact as a large one."""
+    print(f"state gradient rows DK={DK} DV={DV} S={S} decay={decay}", flush=True)
+    ins, s0, do, dh = _inputs(S, 2, DK, DV, decay, S)
+    ref, got = _grads64(ins, s0, do, dh)[6], _grads(ins, s0, do, dh)[6]
+    rows = ref.norm(dim=-1)
+    assert rows.min() < 2.0 ** -10 * rows.max()
+    # a few chained fp32 sums of up to DK + 64 products, as at one magnitude, on factors
+    # e^G whose exponent (up to 150 here, a sum of fp32 decays) is exact to 2^-24 of itself
+    tol = (2 * (DK + 64) + 150) * 2.0 ** -24
+    e = _row_errors(got, ref, 2.0 ** -100).max().item()
+    print(f"  dS0 rows {e:.2e}, {rows.max().log2():.0f} .. {rows.min().log2():.0f}", flush=True)
+    assert e < tol
