@@ -55,3 +55,24 @@ def test_state_gradient_by_channel(S, decay, DK, DV):
     e = _row_errors(got, ref, 2.0 ** -100).max().item()
     print(f"  dS0 rows {e:.2e}, {rows.max().log2():.0f} .. {rows.min().log2():.0f}", flush=True)
     assert e < tol
+
+
+@pytest.mark.parametrize("DK", [32, 64, 128])
+@pytest.mark.parametrize("S,nats", [(16, 5.0), (16, 1.0), (64, 5.1), (70, 4.5)])
+@pytest.mark.parametrize("scale", [1.0, 1e-6, 1e-8])
+def test_small_queries_and_keys_under_decay(scale, S, nats, DK):
+    """dv comes from q and k alone here (no state, no state gradient), by products over
+    16 rows that decay by up to 118 binary orders: relative to its size at any size of q,
+    and as exact near the diagonal as without the decay."""
+    print(f"small queries DK={DK} S={S} nats={nats} scale={scale}", flush=True)
+    ins, s0, do, dh = _inputs(S, 2, DK, 32, 1.0, 7)
+    ins[3] = -nats * (1 + 0.02 * torch.rand(ins[3].shape, generator=torch.Generator().manual_seed(1)))
+    ins[0] = ins[0] * scale
+    s0, dh = torch.zeros_like(s0), torch.zeros_like(dh)
+    ref, got = _grads64(ins, s0, do, dh), _grads(ins, s0, do, dh)
+    # sums of up to DK + 64 products in fp32, their roundings (2^-24) of either sign
+    tol = (DK + 64) ** 0.5 * 2.0 ** -24
+    for i in (2, 5):
+        e = ((got[i] - ref[i]).norm() / ref[i].norm()).item()
+        print(f"  {NAMES[i]} {e:.2e}", flush=True)
+        assert e < tol
