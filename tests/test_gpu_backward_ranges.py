@@ -76,3 +76,32 @@ def test_small_queries_and_keys_under_decay(scale, S, nats, DK):
         e = ((got[i] - ref[i]).norm() / ref[i].norm()).item()
         print(f"  {NAMES[i]} {e:.2e}", flush=True)
         assert e < tol
+
+
+@pytest.mark.parametrize("where", ["q", "k", "v", "do"])
+@pytest.mark.parametrize("S,t,DK,DV,dtype", [(128, 90, 128, 128, torch.float32), (70, 3, 64, 96, torch.bfloat16),
+                                             (64, 40, 32, 48, torch.float16)])
+def test_an_infinity_spoils_only_what_it_reaches(S, t, DK, DV, dtype, where):
+    """One infinite input value: the gradients it is summed into are not finite, and every
+    finite one is what it is without it, not a sum that has lost its other terms."""
+    print(f"infinity in {where} S={S} t={t} DK={DK} DV={DV} {dtype}", flush=True)
+    ins, s0, do, dh = _inputs(S, 2, DK, DV, 0.3, 11)
+    ins = [x if i == 3 else x.to(dtype) for i, x in enumerate(ins)]
+    do = do.to(dtype)
+    want = _grads(ins, s0, do, dh)
+    bad = {"q": 0, "k": 1, "v": 2}.get(where)
+    x = (do if bad is None else ins[bad]).clone()
+    x[0, t, 0, 5] = float("inf")
+    if bad is None:
+        do = x
+    else:
+        ins[bad] = x
+    got = _grads(ins, s0, do, dh)
+    tol = 2 * (DK + 64) * 2.0 ** -24 + {torch.float32: 0, torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}[dtype]
+    for name, a, r in zip(NAMES, got, want):
+        fin = torch.isfinite(a)
+        assert ((a - r).abs()[fin] <= tol * r.abs().max()).all(), name
+        assert fin[..., 1, :].all() if name != "dS0" else fin[:, 1].all(), name     # the other head
+    if where in ("v", "do"):                # a value column of its own in dv, dw and dS_0
+        for i in (2, 5, 6):
+            assert torch.isfinite(torch.cat([got[i][..., :5], got[i][..., 6:]], -1)).all(), NAMES[i]
