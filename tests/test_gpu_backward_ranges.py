@@ -105,3 +105,27 @@ def test_an_infinity_spoils_only_what_it_reaches(S, t, DK, DV, dtype, where):
     if where in ("v", "do"):                # a value column of its own in dv, dw and dS_0
         for i in (2, 5, 6):
             assert torch.isfinite(torch.cat([got[i][..., :5], got[i][..., 6:]], -1)).all(), NAMES[i]
+
+
+@pytest.mark.parametrize("DK,DV", [(64, 64), (128, 128)])
+@pytest.mark.parametrize("bits", [10, 24])
+@pytest.mark.parametrize("state", [False, True])
+def test_rows_far_apart(state, bits, DK, DV):
+    """Rows of d_out and v 2^-10 and 2^-24 of the others' keep their own gradients: row by
+    row as with rows of one size."""
+    print(f"rows far apart DK={DK} DV={DV} bits={bits} state={state}", flush=True)
+    ins, s0, do, dh = _inputs(64, 2, DK, DV, 0.3, 5)
+    do[:, 32:] *= 2.0 ** -bits           # later rows: nothing of a larger one is summed into theirs
+    do[:, 5:17:2] *= 2.0 ** -bits        # (dq_t = d_out_t S^T and its pairs come from row t alone)
+    ins[2][:, 10:30:3] *= 2.0 ** -bits   # dw = v dY
+    dh = torch.zeros_like(dh)
+    s0 = s0 if state else torch.zeros_like(s0)
+    ref, got = _grads64(ins, s0, do, dh), _grads(ins, s0, do, dh)
+    # the largest of 100 rows' sums of up to DK + DV products, roundings of 2^-24: four
+    # standard deviations
+    tol = 4 * (DK + DV) ** 0.5 * 2.0 ** -24
+    for i, name in enumerate(NAMES[:6]):
+        a, r = (got[i], ref[i]) if name not in ("dk", "dg", "db") else (got[i][:, 32:], ref[i][:, 32:])
+        e = _row_errors(a, r, 0).max().item()
+        print(f"  {name} rows {e:.2e}", flush=True)
+        assert e < tol, name
