@@ -223,7 +223,9 @@ int gdn2_hip_gemv(const void* x, long ldx, const void* W, void* y, long ldy, int
  * Chunkwise form in fp32 (chunk 64): per-chunk local factors, a forward scan
  * of the chunk-entry states, a reverse scan of the state gradients, per-chunk
  * gradients, and the sum over the value heads of each key head. DK in {32,
- * 64, 128}, DV a multiple of 16 (<= 4096). `workspace` (256-byte aligned)
+ * 64, 128}, DV a multiple of 16 (<= 4096). Tensors may start at any element (a
+ * 16-bit q, k or b that is not 4-byte aligned is copied into the workspace
+ * first). `workspace` (256-byte aligned)
  * holds gdn2_hip_backward_workspace_bytes(B, H, HK, DK, DV, S) bytes, which
  * grows linearly in B * S: with NC = ceil(S / 64) it is the chunk records
  * (B * HK * NC * 49.3 K floats at DK = 128), two fp32 per-chunk state
