@@ -637,9 +637,13 @@ class GatedDeltaNet2(nn.Module):
     def _trains_fused(self, x):
         """Whether a training pass can take the hip prologue and epilogue in place
         of the torch ops around the op: what the kernels take (one dtype, head
-        sizes, conv width), nothing attached to the modules they stand in for, and no
-        forward-mode differentiation (the torch ops carry tangents, the kernels none)."""
+        sizes, conv width), nothing attached to or overriding the modules and methods
+        they stand in for, and no forward-mode differentiation (the torch ops carry
+        tangents, the kernels none)."""
         DK, DV = self.head_dim_k, self.head_dim_v
+        if any(getattr(type(self), n) is not getattr(GatedDeltaNet2, n) or n in self.__dict__
+               for n in ("_project", "_decay", "_finish")):
+            return False
         if (type(x) is not torch.Tensor or x.dtype not in _hip.DTYPE_CODES or torch.is_autocast_enabled()
                 or forward_ad._current_level >= 0
                 or DK % 8 or DK > 512 or (DK // 8) & (DK // 8 - 1) or DV % 8 or DV > 512 or x.numel() == 0
