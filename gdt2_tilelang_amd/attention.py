@@ -264,6 +264,12 @@ def _unhooked(m, cls):
                      or _nn_module._global_backward_hooks or _nn_module._global_backward_pre_hooks))
 
 
+def _plain(p, shape, device):
+    """An ordinary parameter of this shape and device, as the kernels read it."""
+    return (type(p) in (nn.Parameter, torch.Tensor) and p.shape == shape and p.device == device
+            and p.dtype in _hip.DTYPE_CODES)
+
+
 def gdn2_attention(q, k, v, g, b, w, scale=None, initial_state=None, output_final_state=False,
                    config: GDN2Config = DEFAULT_KERNEL_CONFIG, cu_seqlens=None):
     """Gated DeltaNet-2 attention over a full sequence.
@@ -647,16 +653,22 @@ class GatedDeltaNet2(nn.Module):
         if (type(x) is not torch.Tensor or x.dtype not in _hip.DTYPE_CODES or torch.is_autocast_enabled()
                 or forward_ad._current_level >= 0
                 or DK % 8 or DK > 512 or (DK // 8) & (DK // 8 - 1) or DV % 8 or DV > 512 or x.numel() == 0
-                or not _unhooked(self.o_norm, _GatedRMSNorm)):
+                or x.shape[0] > 65535 or not _unhooked(self.o_norm, _GatedRMSNorm)):
+            return False
+        HK = self.num_kv_heads
+        if not (_plain(self.o_norm.weight, (DV,), x.device) and _plain(self.A_log, (HK,), x.device)
+                and _plain(self.dt_bias, (HK, DK), x.device)):
             return False
         if self.q_conv is not None:
-            convs = (self.q_conv, self.k_conv, self.v_conv)
-            if not 1 <= self.cfg.conv_size <= 4:
+            K = self.cfg.conv_size
+            if not 1 <= K <= 4:
                 return False
-            for c in convs:
+            for c, C in ((self.q_conv, HK * DK), (self.k_conv, HK * DK), (self.v_conv, self.num_heads * DV)):
                 if not (_unhooked(c, _ShortConv) and _unhooked(c.conv, nn.Conv1d) and c.activation
-                        and c.conv.weight.dtype == x.dtype and c.conv.bias is not None
-                        and c.conv.bias.dtype == x.dtype):
+                        and _plain(c.conv.weight, (C, 1, K), x.device) and c.conv.weight.dtype == x.dtype
+                        and _plain(c.conv.bias, (C,), x.device) and c.conv.bias.dtype == x.dtype
+                        and c.conv.padding == (K - 1,) and c.conv.stride == (1,) and c.conv.dilation == (1,)
+                        and c.conv.groups == C and c.conv.padding_mode == "zeros"):
                     return False
         return True
 
@@ -667,8 +679,10 @@ class GatedDeltaNet2(nn.Module):
         HK, H, DK, DV = self.num_kv_heads, self.num_heads, self.head_dim_k, self.head_dim_v
         raw = [p(x) for p in (self.q_proj, self.k_proj, self.v_proj, self.b_proj, self.w_proj, self.f_proj)]
         gate = self.o_gate_proj(x)
-        if any(type(t) is not torch.Tensor or t.dtype != x.dtype for t in (*raw, gate)):
-            # a replaced projection: the torch ops take what it gave
+        if any(type(t) is not torch.Tensor or t.dtype != x.dtype or t.device != x.device
+               or t.shape != (B, S, n) for t, n in zip((*raw, gate), [HK * DK, HK * DK, H * DV, HK * DK, H * DV, HK * DK,
+                                                                        H * DV])):
+            # a replaced projection: the torch ops take, or refuse, what it gave
             o, final_state = gdn2_attention(*self._project(x, None, raw), scale=self.scale,
                                             initial_state=initial_state, output_final_state=use_cache,
                                             config=self.cfg.kernel)
