@@ -646,7 +646,7 @@ __global__ __launch_bounds__(kThreads) void epilogue_bwd_kernel(const void* __re
       const float sg = sigmoid(gt[e]), sl = gt[e] * sg;
       dx[e] = r * w[e] * sl * d[e] - k * x[e];
       dgt[e] = x[e] * r * w[e] * d[e] * sg * (1.f + gt[e] * (1.f - sg));
-      gw[e] += x[e] * r * sl * d[e];
+      if (act) gw[e] += x[e] * r * sl * d[e];   // (a lane past the rows has r = 1 / sqrt(eps), infinite for eps = 0)
     }
     if (act) {
       st8<ODT>(d_o, at, dx);
