@@ -192,7 +192,7 @@ def bench_varlen(reps=20, nseq=16):
 
 
 def bench_backward(reps=5):
-    """Training backward at config 1's shape (bf16 inputs, fp32 arithmetic):
+    """Training backward at config 1's shape (bf16 inputs, fp32 sums, split-fp16 products):
     chunk_gdn2_bwd with no initial state and no final-state gradient, the
     common training case; timed with HIP events on the current stream."""
     from gdt2_tilelang_amd import chunk_gdn2_bwd
@@ -211,7 +211,7 @@ def bench_backward(reps=5):
     torch.cuda.synchronize()
     ms = e0.elapsed_time(e1) / reps
     return {"workload": "chunk_gdn2_bwd, BASELINE config 1 shape (B=2 S=4096 H=16 DK=DV=128, bf16 in, fp32 "
-                        "arithmetic, dq dk dv dg db dw)", "ms": round(ms, 3),
+                        "sums, split-fp16 products, dq dk dv dg db dw)", "ms": round(ms, 3),
             "tokens_per_s": round(B1 * S1 / (ms * 1e-3), 1), "reps": reps}
 
 

@@ -639,9 +639,15 @@ static hipError_t launch_scan_e_t(const void* v, const void* w, const unsigned s
 // workgroup's LDS fills a CU): half the rounds at 1.3 times the step. 8 x 16 heads x 8
 // tiles of 4000 tokens: 344 us in four rounds of one tile, 206 in two of two. At or
 // below one round the shorter step wins: 256 tiles of 4096 tokens 81 us against 96,
-// 128 tiles of 8175 127 against 171. A packed batch's longest sequence may outlast the
-// others' rounds, and its length is on the device only: three rounds' worth of
-// tiles are asked for there (16 prompts of 8192 tokens, 2048 tiles: 121 us -> 79).
+// 128 tiles of 8175 127 against 171. A packed batch runs as long as its longest
+// sequence, whose length the C entry has on the device only: three rounds' worth of
+// tiles are asked for there. Whole forward calls of 8192 tokens, one tile against two,
+// with equal lengths, with one sequence of half the tokens, and of 95% of them:
+//   512 tiles  167 / 140 us   193 / 177   226 / 233
+//   768        183 / 165      203 / 194   233 / 242
+//   1024       177 / 144      212 / 192   236 / 241
+//   2048       200 / 154      240 / 210   260 / 253
+// (16 prompts of random lengths, 2048 tiles: the scan 121 -> 79 us.)
 static bool sce_two_tiles(int B, int H, int DV, bool packed) {
   constexpr long kCUs = 256;
   return DV % (2 * sce::DVT) == 0 && static_cast<long>(B) * H * (DV / sce::DVT) > (packed ? 3 * kCUs : kCUs);

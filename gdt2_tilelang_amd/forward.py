@@ -166,10 +166,11 @@ def chunk_gdn2_bwd(q, k, v, g, b, w, scale, initial_state, do, dht, config: GDN2
     gradients of ``(o * do).sum() + (final_state * dht).sum()`` with respect
     to the forward inputs. Returns ``(dq, dk, dv, dg, db, dw, dinitial_state)``;
     the last is ``None`` when ``initial_state`` is ``None``. Each gradient has
-    its input's dtype. The arithmetic is fp32 throughout (chunk 64):
-    ``gdn2_hip_backward`` recomputes the per-chunk factors, scans the
-    chunk-entry states forward and the state gradients backward, then forms
-    every chunk's gradients in parallel.
+    its input's dtype. Sums, states and intermediate arrays are fp32 (chunk
+    64); matrix products take fp32 operands as fp16 high and low parts, 22 to
+    23 significant bits (``gdn2_backward.hip``). ``gdn2_hip_backward``
+    recomputes the per-chunk factors, scans the chunk-entry states forward and
+    the state gradients backward, then forms every chunk's gradients in parallel.
     """
     dev = _require_device(q, k, v, g, b, w, do)
     _check_shapes(q, k, v, g, b, w)

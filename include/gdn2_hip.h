@@ -220,7 +220,8 @@ int gdn2_hip_gemv(const void* x, long ldx, const void* W, void* y, long ldy, int
  *   dg [B, S, HK, DK] fp32, and, if d_initial_state is not null, the
  *   gradient of initial_state (fp32 [B, H, DK, DV]; null initial_state means
  *   zeros) into d_initial_state.
- * Chunkwise form in fp32 (chunk 64): per-chunk local factors, a forward scan
+ * Chunkwise form (chunk 64) with fp32 sums, states and intermediate arrays and
+ * split-fp16 operands (22 to 23 bits) in the products: per-chunk local factors, a forward scan
  * of the chunk-entry states, a reverse scan of the state gradients, per-chunk
  * gradients, and the sum over the value heads of each key head. DK in {32,
  * 64, 128}, DV a multiple of 16 (<= 4096). Tensors may start at any element (a
@@ -257,7 +258,7 @@ int gdn2_hip_backward(const void* q, const void* k, const void* v, const float* 
  * All sequences run in one set of launches: the per-chunk kernels take the
  * forward's record slots (chunk c of sequence s at slot s + floor(cu[s]/64)
  * + c; slots between sequences exit at once) and the scans run per
- * (sequence, value head, 16 columns). Workspace (256-byte aligned):
+ * (sequence, value head, 16 or 32 columns). Workspace (256-byte aligned):
  * gdn2_hip_backward_varlen_workspace_bytes, the dense formula with
  * ceil(T/64) + nseq chunk slots per head.
  * No reference counterpart: the reference raises for cu_seqlens

@@ -85,5 +85,5 @@ def test_packed_offsets_are_the_calls_own(where, dtype):
         assert torch.equal(o[:, a:e], oo)
         for t, d in zip(want, torch.autograd.grad(oo.sum() + ss.sum(), part)):
             t[:, a:e] = d
-    for x, y in zip(got, want):   # the same kernels on the same rows; only the weights' reductions may regroup
+    for x, y in zip(got, want):   # the same kernels on the same rows, in chunks that start at the same tokens
         assert (x - y).norm() <= 1e-6 * y.norm()
